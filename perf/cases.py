@@ -19,7 +19,6 @@ import random
 import torch
 
 from tread_amd import BlockStore, Engine, _hip, blend
-from tread_amd.forward import alloc_cache
 from tread_amd.model import preset, synthetic_model
 
 SYSTEM = 64  # tokens of the system prompt that every request shape of this repository starts with
