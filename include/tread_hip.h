@@ -202,6 +202,37 @@ size_t tread_skinny_silu_workspace_bytes(int64_t m, int64_t n, int64_t inter);
 int tread_skinny_silu_linear_bf16(const void* gate_up, int64_t m, int64_t inter, const void* weight, int64_t n, void* y,
                                   void* ws, size_t ws_bytes, tread_stream_t stream);
 
+/* Linear layer of up to 64 token rows: y[m, n] = x[m, k] . weight[n, k]^T (+ bias[n]), bf16, fp32
+ * accumulation, one bf16 rounding (as F.linear); x, y and weight contiguous and 16-byte aligned, n a
+ * multiple of 64, k of 128. The weights are streamed once, cut into equal spans over the GPU; the
+ * spans' fp32 sums meet in ws (device, tread_mid_linear_workspace_bytes(m, n, k) bytes, required; 0
+ * bytes: the shape is not supported).
+ */
+size_t tread_mid_linear_workspace_bytes(int64_t m, int64_t n, int64_t k);
+int tread_mid_linear_bf16(const void* x, const void* weight, const void* bias, int64_t m, int64_t n, int64_t k, void* y,
+                          void* ws, size_t ws_bytes, tread_stream_t stream);
+
+/* n_layers consecutive decoder layers for m <= 64 token rows (the query forward of
+ * tread/engine.py:131-132, a short prefill), every kernel queued by one call: per layer add +
+ * RMSNorm, q|k|v, RoPE + splice of k/v into rows rows[i] of the layer's cache, attention
+ * (tread_subset_attn_bf16's row semantics: kend, kseg, n_shared), o, add + RMSNorm, gate|up, SiLU
+ * gating, down, with the roundings of the single entry points. h, delta (may be NULL), h_out,
+ * delta_out: [m, hidden]; h_out and delta_out are the residual stream and pending MLP output after
+ * the last layer. All device pointers 16-byte aligned; ws: device,
+ * tread_mid_layers_workspace_bytes(...) bytes (0: the shape is not supported).
+ */
+typedef struct {
+  const void *ln1, *wqkv, *bqkv; /* bqkv may be NULL */
+  const void *wo, *ln2, *wgu, *wd;
+  void *k_cache, *v_cache; /* [hkv, t_cap, head_dim] */
+} tread_layer_t;
+size_t tread_mid_layers_workspace_bytes(int64_t m, int hidden, int hq, int hkv, int head_dim, int inter, int64_t t_cap);
+int tread_mid_layers_bf16(const tread_layer_t* layers, int n_layers, const void* h, const void* delta, int64_t m,
+                          int hidden, int hq, int hkv, int head_dim, int inter, float eps, const void* cos,
+                          const void* sin, const int64_t* rows, const int64_t* kend, const int64_t* kseg,
+                          int64_t n_shared, int64_t t_cap, float scale, void* h_out, void* delta_out, void* ws,
+                          size_t ws_bytes, tread_stream_t stream);
+
 /* ---------------------------------------------------------------------------------------------
  * (d) Block-tier copy: async DMA of `bytes` between pinned host and device memory (either
  * direction) on `stream`, then records `done` (may be NULL) on the same stream.

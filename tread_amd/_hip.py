@@ -10,11 +10,16 @@ from pathlib import Path
 import torch  # loads torch's HIP runtime first, so the library below binds to the same one
 
 LIB_PATH = Path(__file__).resolve().with_name("libtread_hip.so")
-ABI_VERSION = 10
+ABI_VERSION = 11
 
 c_i64, c_int, c_void, c_float, c_size = ctypes.c_int64, ctypes.c_int, ctypes.c_void_p, ctypes.c_float, ctypes.c_size_t
 P_I64 = ctypes.POINTER(ctypes.c_int64)
 P_F32 = ctypes.POINTER(ctypes.c_float)
+
+
+class Layer(ctypes.Structure):
+    """tread_layer_t."""
+    _fields_ = [(n, c_void) for n in ("ln1", "wqkv", "bqkv", "wo", "ln2", "wgu", "wd", "k_cache", "v_cache")]
 
 
 class Src(ctypes.Structure):
@@ -53,6 +58,12 @@ _SIGS = {
                                               c_void, c_void]),
     "tread_skinny_silu_workspace_bytes": (c_size, [c_i64, c_i64, c_i64]),
     "tread_skinny_silu_linear_bf16": (c_int, [c_void, c_i64, c_i64, c_void, c_i64, c_void, c_void, c_size, c_void]),
+    "tread_mid_linear_workspace_bytes": (c_size, [c_i64, c_i64, c_i64]),
+    "tread_mid_linear_bf16": (c_int, [c_void, c_void, c_void, c_i64, c_i64, c_i64, c_void, c_void, c_size, c_void]),
+    "tread_mid_layers_workspace_bytes": (c_size, [c_i64, c_int, c_int, c_int, c_int, c_int, c_i64]),
+    "tread_mid_layers_bf16": (c_int, [ctypes.POINTER(Layer), c_int, c_void, c_void, c_i64, c_int, c_int, c_int, c_int,
+                                      c_int, c_float, c_void, c_void, c_void, c_void, c_void, c_i64, c_i64, c_float,
+                                      c_void, c_void, c_void, c_size, c_void]),
     "tread_copy_async": (c_int, [c_void, c_void, c_size, c_void, c_void]),
     "tread_copy_layers_async": (c_int, [c_void, c_void, c_void, c_int, c_int, c_void, c_void]),
 }
@@ -345,6 +356,81 @@ def skinny_silu_linear(gate_up, weight):
     _check("tread_skinny_silu_linear_bf16", lib().tread_skinny_silu_linear_bf16(
         _ptr(gate_up), m, inter, _ptr(weight), n, _ptr(y), _ptr(ws), wsb, _stream()))
     return y
+
+
+MID_MAX_ROWS = 64
+
+
+def mid_linear(x, weight, bias=None):
+    """y = x @ weight.T (+ bias) for x [m, k], m <= 64: the weight-streaming kernel of mid_layers."""
+    _need(x, "x")
+    _need(weight, "weight")
+    if bias is not None:
+        _need(bias, "bias")
+    m, k = x.shape
+    n = weight.shape[0]
+    wsb = lib().tread_mid_linear_workspace_bytes(m, n, k)
+    if weight.shape[1] != k or not wsb:
+        raise ValueError(f"mid_linear: unsupported shape x {tuple(x.shape)} weight {tuple(weight.shape)}")
+    y = torch.empty(m, n, dtype=x.dtype, device=x.device)
+    ws = torch.empty(wsb, dtype=torch.uint8, device=x.device)
+    _check("tread_mid_linear_bf16", lib().tread_mid_linear_bf16(
+        _ptr(x), _ptr(weight), _ptr(bias), m, n, k, _ptr(y), _ptr(ws), wsb, _stream()))
+    return y
+
+
+def mid_layers_ok(m, H, hq, hkv, hd, inter):
+    """Layers mid_layers takes (rows <= 64, widths in whole 64-feature by 128-wide units)."""
+    return 0 < m <= MID_MAX_ROWS and lib().tread_mid_layers_workspace_bytes(m, H, hq, hkv, hd, inter, 1) > 0
+
+
+def mid_layers(layers, caches, h, delta, eps, hq, hkv, hd, inter, cos, sin, rows, kend, scale, kseg=None, n_shared=0):
+    """Consecutive decoder layers for m <= 64 rows h [m, H] (residual h + delta, delta may be None),
+    queued by one library call. layers: model.LayerW per layer; caches: (K, V) of each, one layer
+    [(1,) hkv, t_cap, hd]. Returns (h, delta) after the last layer."""
+    _need(h, "h")
+    if delta is not None:
+        _need(delta, "delta")
+        if delta.shape != h.shape:
+            raise ValueError("mid_layers: delta shape differs from h")
+    m, H = h.shape
+    n_qkv = (hq + 2 * hkv) * hd
+    t_cap = caches[0][0].shape[-2]
+    for t, name in ((rows, "rows"), (kend, "kend"), (kseg, "kseg")):
+        if t is not None:
+            _need(t, name, torch.int64)
+            if t.numel() != m:
+                raise ValueError(f"mid_layers: {name} has {t.numel()} entries for {m} rows")
+    for t, name in ((cos, "cos"), (sin, "sin")):
+        _need(t, name)
+        if t.shape != (m, hd // 2):
+            raise ValueError(f"mid_layers: {name} must be [{m}, {hd // 2}]")
+    arr = (Layer * len(layers))()
+    for i, (lw, (K, V)) in enumerate(zip(layers, caches)):
+        for t, name, shape in ((lw.ln1, "ln1", (H,)), (lw.wqkv, "wqkv", (n_qkv, H)), (lw.bqkv, "bqkv", (n_qkv,)),
+                               (lw.wo, "wo", (H, hq * hd)), (lw.ln2, "ln2", (H,)), (lw.wgu, "wgu", (2 * inter, H)),
+                               (lw.wd, "wd", (H, inter))):
+            if t is None and name == "bqkv":
+                continue
+            _need(t, name)
+            if t.shape != shape:
+                raise ValueError(f"mid_layers: layer {i} {name} {tuple(t.shape)}, expected {shape}")
+        for t, name in ((K, "k_cache"), (V, "v_cache")):
+            _need(t, name)
+            if t.numel() != hkv * t_cap * hd or t.shape[-2:] != (t_cap, hd):
+                raise ValueError(f"mid_layers: layer {i} {name} {tuple(t.shape)}")
+        arr[i] = Layer(lw.ln1.data_ptr(), lw.wqkv.data_ptr(), None if lw.bqkv is None else lw.bqkv.data_ptr(),
+                       lw.wo.data_ptr(), lw.ln2.data_ptr(), lw.wgu.data_ptr(), lw.wd.data_ptr(), K.data_ptr(),
+                       V.data_ptr())
+    wsb = lib().tread_mid_layers_workspace_bytes(m, H, hq, hkv, hd, inter, t_cap)
+    if not wsb:
+        raise ValueError(f"mid_layers: unsupported shape m={m} H={H} hq={hq} hkv={hkv} hd={hd} inter={inter}")
+    ws = torch.empty(wsb, dtype=torch.uint8, device=h.device)
+    h_out, d_out = torch.empty_like(h), torch.empty_like(h)
+    _check("tread_mid_layers_bf16", lib().tread_mid_layers_bf16(
+        arr, len(layers), _ptr(h), _ptr(delta), m, H, hq, hkv, hd, inter, float(eps), _ptr(cos), _ptr(sin), _ptr(rows),
+        _ptr(kend), _ptr(kseg), int(n_shared), t_cap, float(scale), _ptr(h_out), _ptr(d_out), _ptr(ws), wsb, _stream()))
+    return h_out, d_out
 
 
 def silu_mul(gate_up, out=None):

@@ -28,11 +28,10 @@
 // Few rows (the query forward: tens of rows over a long cache) would leave most CUs idle, so the
 // key range is then split across work groups (split-K): each writes its unnormalised fp32 O and
 // its running (max, sum) to a workspace, and a combine kernel merges the splits per row.
-#include <utility>
-
 #include <mutex>
 
 #include "common.h"
+#include "lds.h"
 #include "../../include/tread_hip.h"
 
 namespace tread {
@@ -101,12 +100,6 @@ __device__ __forceinline__ s16x4_t lds_read_tr16(const bf16_t* p) {
       (__attribute__((address_space(3))) s16x4_t*)((__attribute__((address_space(3))) char*)(uintptr_t)p));
 }
 
-// 16 bytes per lane from global memory straight into LDS: lane l's bytes land at lds + 16 l
-// (lds is wave-uniform).
-__device__ __forceinline__ void lds_load16(const bf16_t* g, bf16_t* lds) {
-  __builtin_amdgcn_global_load_lds(g, (__attribute__((address_space(3))) void*)(uintptr_t)lds, 16, 0, 0);
-}
-
 constexpr float ATT_RESCALE_LOG2 = 8.0f;  // keep a stale row max until it is 2^8 too small
 
 __device__ __forceinline__ int wave_max(int v) {
@@ -130,10 +123,6 @@ __device__ __forceinline__ int wave_min(int v) {
   return v;
 }
 
-// LDS byte address of a pointer into the work group's shared memory (the low 32 bits of its
-// generic address; the LDS aperture is 4 GiB-aligned).
-__device__ __forceinline__ uint32_t lds_addr(const void* p) { return (uint32_t)(uintptr_t)p; }
-
 // V^T fragment halves by inline asm rather than the intrinsic: the compiler would otherwise wait
 // for every outstanding global->LDS load (the next tiles' prefetch) before the first transposing
 // read of a tile. The caller orders the results with lgkm_wait before use.
@@ -156,37 +145,6 @@ __device__ __forceinline__ void lgkm_wait(s16x4_t (&v)[M]) {
   else
     asm volatile("s_waitcnt lgkmcnt(%4)" : "+v"(v[0]), "+v"(v[1]), "+v"(v[2]), "+v"(v[3]) : "n"(N));
 }
-
-template <int OFF>
-__device__ __forceinline__ bf16x8_t lds_read128(uint32_t addr) {
-  u32x4_t r;
-  asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(r) : "v"(addr), "n"(OFF));
-  return __builtin_bit_cast(bf16x8_t, r);
-}
-template <int N>
-__device__ __forceinline__ void lgkm_wait(bf16x8_t& v) {
-  asm volatile("s_waitcnt lgkmcnt(%1)" : "+v"(v) : "n"(N));
-}
-
-template <int... I, typename F>
-__device__ __forceinline__ void static_for_impl(std::integer_sequence<int, I...>, F&& f) {
-  (f(std::integral_constant<int, I>{}), ...);
-}
-template <int N, typename F>
-__device__ __forceinline__ void static_for(F&& f) {
-  static_for_impl(std::make_integer_sequence<int, N>{}, f);
-}
-
-template <int N>
-__device__ __forceinline__ void vm_wait() {
-  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
-}
-
-// Work-group barrier of the tile pipelines, after each wave has waited (vm_wait) for its own
-// global->LDS loads of the tiles the barrier publishes. __syncthreads() would also wait for every
-// outstanding vector memory operation (vmcnt(0)), i.e. for the tiles still being prefetched,
-// taking the pipeline's load lead away at every barrier.
-__device__ __forceinline__ void tile_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
 // max over lanes l and l ^ 32 (the two key halves of one query column)
 __device__ __forceinline__ float xhalf_max(float v) {
@@ -1174,21 +1132,6 @@ constexpr int DEC_MIN_SPLIT = 4 * DEC_BK;
 // causal pass).
 constexpr int ATT_LONG_MIN_TILES = 8;
 constexpr int64_t ATT_LONG_MAX_WGS = 1536;
-
-// Compute units of the current device, looked up once per device.
-static int cu_count() {
-  static std::mutex mu;
-  static int cache[64];
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
-  std::lock_guard<std::mutex> lock(mu);
-  if (!cache[dev]) {
-    int v = 0;
-    if (hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || v <= 0) v = 256;
-    cache[dev] = v;
-  }
-  return cache[dev];
-}
 
 static SplitPlan plan_split(int64_t n, int hq, int hkv, int head_dim, int64_t t_cap) {
   SplitPlan sp;

@@ -115,6 +115,7 @@ namespace tread {
 void set_error(const char* fmt, ...);
 int fail(int code, const char* fmt, ...);
 int check_launch(const char* what);
+int cu_count();  // compute units of the current device
 }  // namespace tread
 
 #define TREAD_EINVAL (-22)

@@ -2,6 +2,8 @@
 #include <stdarg.h>
 #include <stdio.h>
 
+#include <mutex>
+
 #include "common.h"
 #include "../../include/tread_hip.h"
 
@@ -30,11 +32,26 @@ int check_launch(const char* what) {
   return 0;
 }
 
+// Compute units of the current device, looked up once per device.
+int cu_count() {
+  static std::mutex mu;
+  static int cache[64];
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
+  std::lock_guard<std::mutex> lock(mu);
+  if (!cache[dev]) {
+    int v = 0;
+    if (hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || v <= 0) v = 256;
+    cache[dev] = v;
+  }
+  return cache[dev];
+}
+
 }  // namespace tread
 
 extern "C" const char* tread_last_error(void) { return tread::g_err; }
 
-extern "C" int tread_abi_version(void) { return 10; }
+extern "C" int tread_abi_version(void) { return 11; }
 
 extern "C" int tread_copy_layers_async(void* const* dst, const void* const* src, const size_t* bytes, int per_layer,
                                        int n_layers, tread_stream_t stream, const tread_event_t* layer_done) {

@@ -69,6 +69,8 @@ def layer_forward(P, l, h, delta, R: Rows, K, V, kv_only=False):
     hq, hkv, hd = P.hq, P.hkv, P.hd
     if not kv_only and _few_rows(P, lw, h.shape[0]):
         return _layer_few_rows(P, l, lw, h, delta, R, K, V)
+    if not kv_only and _mid_rows(P, h.shape[0]):
+        return _layers_mid_rows(P, [l], h, delta, R, K, V)
     h, x = _hip.add_rmsnorm(h, lw.ln1, P.eps, delta=delta)
     n = h.shape[0]
     if kv_only:
@@ -144,12 +146,26 @@ def _layer_few_rows(P, l, lw, h, delta, R, K, V):
     return h, _silu_linear(gu, lw.wd)
 
 
+def _mid_rows(P, n):
+    return FEW_ROWS < n <= _hip.MID_MAX_ROWS and _hip.mid_layers_ok(n, P.H, P.hq, P.hkv, P.hd, P.inter)
+
+
+def _layers_mid_rows(P, layers, h, delta, R, K, V):
+    """layer_forward of consecutive layers for 9 to 64 rows, in one library call."""
+    return _hip.mid_layers([P.layers[l] for l in layers], [(K[l], V[l]) for l in layers], h, delta, P.eps, P.hq, P.hkv,
+                           P.hd, P.inter, R.cos, R.sin, R.rows, R.kend, P.scale, kseg=R.kseg, n_shared=R.n_shared)
+
+
 def run_layers(P, h, delta, R, K, V, layers, kv_only_last=False, hook=None, keep=None):
     """Run `layers` (an ordered range) for rows R; `hook(l)` runs before layer l (lazy assembly).
     With kv_only_last, the last layer only splices its k/v (its hidden output is never used),
     except for the rows at positions `keep` (int64 tensor), which then run it fully after every
     row's k/v is in place; the result is those rows' (h, delta)."""
     layers = list(layers)
+    whole = layers[:-1] if kv_only_last else layers
+    if hook is None and whole and _mid_rows(P, h.shape[0]):  # nothing waits between layers
+        h, delta = _layers_mid_rows(P, whole, h, delta, R, K, V)
+        layers = layers[len(whole):]
     for j, l in enumerate(layers):
         if hook is not None:
             hook(l)
