@@ -202,7 +202,7 @@ size_t tread_skinny_silu_workspace_bytes(int64_t m, int64_t n, int64_t inter);
 int tread_skinny_silu_linear_bf16(const void* gate_up, int64_t m, int64_t inter, const void* weight, int64_t n, void* y,
                                   void* ws, size_t ws_bytes, tread_stream_t stream);
 
-/* Linear layer of up to 64 token rows: y[m, n] = x[m, k] . weight[n, k]^T (+ bias[n]), bf16, fp32
+/* Linear layer of up to 128 token rows: y[m, n] = x[m, k] . weight[n, k]^T (+ bias[n]), bf16, fp32
  * accumulation, one bf16 rounding (as F.linear); x, y and weight contiguous and 16-byte aligned, n a
  * multiple of 64, k of 128. The weights are streamed once, cut into equal spans over the GPU; the
  * spans' fp32 sums meet in ws (device, tread_mid_linear_workspace_bytes(m, n, k) bytes, required; 0
@@ -212,7 +212,7 @@ size_t tread_mid_linear_workspace_bytes(int64_t m, int64_t n, int64_t k);
 int tread_mid_linear_bf16(const void* x, const void* weight, const void* bias, int64_t m, int64_t n, int64_t k, void* y,
                           void* ws, size_t ws_bytes, tread_stream_t stream);
 
-/* n_layers consecutive decoder layers for m <= 64 token rows (the query forward of
+/* n_layers consecutive decoder layers for m <= 128 token rows (the query forward of
  * tread/engine.py:131-132, a short prefill), every kernel queued by one call: per layer add +
  * RMSNorm, q|k|v, RoPE + splice of k/v into rows rows[i] of the layer's cache, attention
  * (tread_subset_attn_bf16's row semantics: kend, kseg, n_shared), o, add + RMSNorm, gate|up, SiLU

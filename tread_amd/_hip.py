@@ -358,11 +358,11 @@ def skinny_silu_linear(gate_up, weight):
     return y
 
 
-MID_MAX_ROWS = 64
+MID_MAX_ROWS = 128
 
 
 def mid_linear(x, weight, bias=None):
-    """y = x @ weight.T (+ bias) for x [m, k], m <= 64: the weight-streaming kernel of mid_layers."""
+    """y = x @ weight.T (+ bias) for x [m, k], m <= 128: the weight-streaming kernel of mid_layers."""
     _need(x, "x")
     _need(weight, "weight")
     if bias is not None:
@@ -380,12 +380,12 @@ def mid_linear(x, weight, bias=None):
 
 
 def mid_layers_ok(m, H, hq, hkv, hd, inter):
-    """Layers mid_layers takes (rows <= 64, widths in whole 64-feature by 128-wide units)."""
+    """Layers mid_layers takes (rows <= 128, widths in whole 64-feature by 128-wide units)."""
     return 0 < m <= MID_MAX_ROWS and lib().tread_mid_layers_workspace_bytes(m, H, hq, hkv, hd, inter, 1) > 0
 
 
 def mid_layers(layers, caches, h, delta, eps, hq, hkv, hd, inter, cos, sin, rows, kend, scale, kseg=None, n_shared=0):
-    """Consecutive decoder layers for m <= 64 rows h [m, H] (residual h + delta, delta may be None),
+    """Consecutive decoder layers for m <= 128 rows h [m, H] (residual h + delta, delta may be None),
     queued by one library call. layers: model.LayerW per layer; caches: (K, V) of each, one layer
     [(1,) hkv, t_cap, hd]. Returns (h, delta) after the last layer."""
     _need(h, "h")

@@ -48,6 +48,8 @@ constexpr int ATT_NBUF = 3;                    // LDS tile buffers (software pip
 constexpr int N_XCD = 8;
 constexpr int ATT_TARGET_WGS = 512;     // split-K when fewer (head, row tile) work groups than this
 constexpr int ATT_MIN_SPLIT_KEYS = 512;
+// fewest keys per split below ATT_MANY_TILE_WGS work groups, in whole key tiles
+constexpr int att_few_split_keys(int head_dim) { return head_dim == 64 ? 128 : 192; }
 constexpr int ATT_MANY_TILE_WGS = 64;   // (head, row tile) work groups from which the split aims higher
 
 struct AttnArgs {
@@ -219,6 +221,16 @@ __global__ __launch_bounds__(ATT_THREADS) void subset_attn_kernel(const AttnArgs
     smax = smin = my_seg;
   }
 
+  // Q is loaded beside the key ends (one round of memory latency before the first tile goes out, not
+  // two: 7B query rows 25.9 -> 25.3 us over 3 000 keys, 66.3 -> 64.8 over 32 000). A lane past the
+  // rows reads row 0; its column's scores and output are never used.
+  u32x4_t qraw[KS];
+  {
+    const bf16_t* qp = a.q + (qi * a.hq + qh) * HD + half * 8;
+#pragma unroll
+    for (int s = 0; s < KS; ++s) qraw[s] = *reinterpret_cast<const u32x4_t*>(qp + s * 16);
+  }
+
   // ---- work-group key range
   {
     vmax = wave_max(vmax);
@@ -265,11 +277,9 @@ __global__ __launch_bounds__(ATT_THREADS) void subset_attn_kernel(const AttnArgs
   // the MFMA, started from -m_run, yields the exponent of exp2 directly
   bf16x8_t qf[KS];
   {
-    const bf16_t* qp = a.q + (qi * a.hq + qh) * HD + half * 8;
 #pragma unroll
     for (int s = 0; s < KS; ++s) {
-      u32x4_t t = {0, 0, 0, 0};
-      if (valid) t = *reinterpret_cast<const u32x4_t*>(qp + s * 16);
+      u32x4_t t = qraw[s];
 #pragma unroll
       for (int w = 0; w < 4; ++w) t[w] = pack_bf(lo_bf(t[w]) * a.scale_log2, hi_bf(t[w]) * a.scale_log2);
       qf[s] = __builtin_bit_cast(bf16x8_t, t);
@@ -1154,33 +1164,43 @@ static SplitPlan plan_split(int64_t n, int hq, int hkv, int head_dim, int64_t t_
   sp.nsplit = 1;
   sp.split_len = 0;
   sp.nlong = 0;
-  if (base < ATT_TARGET_WGS && t_cap >= 2 * ATT_MIN_SPLIT_KEYS) {
-    const bool many = base >= ATT_MANY_TILE_WGS;
-    int64_t want = (ATT_TARGET_WGS + base - 1) / base;
-    if (many) {
-      // Many row tiles with ragged key ranges (recompute rows sorted by position): about three
-      // work groups per CU over the launch, rounded, skipping multiples of 4; none when the row
-      // tiles alone fill the CUs (then whole tiles, the longest in key halves). Swept in whole
-      // requests on MI355X (deviation-selected rows, graph buckets, TTFT in one process): 0.5B 8k
-      // (100 row-tile groups) 8.10 / 7.01 / 6.46 / 6.36 / 6.28 / 6.45 / 6.43 ms with 2 / 3 / 5 /
-      // 6 / 7 / 9 / 11 slices, 1.5B 16k (158 groups) 21.76 / 19.63 / 19.42 / 19.94 / 19.74 /
-      // 19.95 ms with 2 / 3 / 5 / 6 / 7 / 9; slice counts that are multiples of 4 were slow on
-      // every shape swept. The 0.5B deviation pass (438 groups) ran 245 us in 3 slices and 201 us
-      // in whole tiles with key halves.
-      const int64_t cus = cu_count();
-      want = base >= cus ? 1 : (6 * cus / base + 1) / 2;
-      if (want >= 4 && want % 4 == 0) --want;
+  const int64_t cus = cu_count(), bk = att_bk(head_dim);
+  int64_t len = 0;  // keys per split (0: no split)
+  if (base < ATT_MANY_TILE_WGS) {
+    // Few row tiles (a query, a short turn): at most one work group per CU, since each holds most of
+    // a CU's LDS and a few more would run as a second round, but as few keys each as that allows.
+    // The split points then do not depend on t_cap until the CUs are used up: a context gives the
+    // same bits in a cache of its own size and in a larger one (but for a last slice of under 32
+    // keys, which is not worth a merge). Against up to 512 work groups of at
+    // least 512 keys (32 rows, time of the call): 0.5B over 1 100 keys 19.4 -> 12.9 us, over 8 100
+    // 23.5 -> 16.2, 1.5B 24.8 -> 18.5 and 27.6 -> 20.5, 7B 25.8 -> 20.0 and 32.3 -> 26.7; 70B over
+    // 32 000 74.7 -> 57.4 (there 512 work groups ran as two rounds).
+    const int64_t most = cus / base;  // splits
+    if (most > 1) {
+      len = (t_cap + most - 1) / most;
+      if (len < att_few_split_keys(head_dim)) len = att_few_split_keys(head_dim);
+      if (t_cap < len + 32) len = 0;
     }
-    int64_t most = t_cap / (many ? 2 * ATT_MIN_SPLIT_KEYS : ATT_MIN_SPLIT_KEYS);
-    int64_t ns = want < most ? want : most;
-    if (ns > CMB_MAX_SPLITS) ns = CMB_MAX_SPLITS;
-    if (ns > 1) {
-      int64_t len = (t_cap + ns - 1) / ns;
-      const int64_t bk = att_bk(head_dim);
-      len = (len + bk - 1) / bk * bk;
-      sp.nsplit = (int)((t_cap + len - 1) / len);
-      sp.split_len = (int)len;
-    }
+  } else if (base < ATT_TARGET_WGS && t_cap >= 2 * ATT_MIN_SPLIT_KEYS) {
+    // Many row tiles with ragged key ranges (recompute rows sorted by position): about three
+    // work groups per CU over the launch, rounded, skipping multiples of 4; none when the row
+    // tiles alone fill the CUs (then whole tiles, the longest in key halves). Swept in whole
+    // requests on MI355X (deviation-selected rows, graph buckets, TTFT in one process): 0.5B 8k
+    // (100 row-tile groups) 8.10 / 7.01 / 6.46 / 6.36 / 6.28 / 6.45 / 6.43 ms with 2 / 3 / 5 /
+    // 6 / 7 / 9 / 11 slices, 1.5B 16k (158 groups) 21.76 / 19.63 / 19.42 / 19.94 / 19.74 /
+    // 19.95 ms with 2 / 3 / 5 / 6 / 7 / 9; slice counts that are multiples of 4 were slow on
+    // every shape swept. The 0.5B deviation pass (438 groups) ran 245 us in 3 slices and 201 us
+    // in whole tiles with key halves.
+    int64_t want = base >= cus ? 1 : (6 * cus / base + 1) / 2;
+    if (want >= 4 && want % 4 == 0) --want;
+    const int64_t most = t_cap / (2 * ATT_MIN_SPLIT_KEYS);
+    const int64_t ns = want < most ? want : most;
+    if (ns > 1) len = (t_cap + ns - 1) / ns;
+  }
+  if (len > 0) {
+    len = (len + bk - 1) / bk * bk;
+    sp.nsplit = (int)((t_cap + len - 1) / len);
+    sp.split_len = sp.nsplit > 1 ? (int)len : 0;
   }
   if (sp.nsplit == 1 && sp.tiles >= ATT_LONG_MIN_TILES && base <= ATT_LONG_MAX_WGS) sp.nlong = (int)((sp.tiles + 2) / 4);
   return sp;

@@ -12,6 +12,11 @@ __device__ __forceinline__ void lds_load16(const bf16_t* g, bf16_t* lds) {
   __builtin_amdgcn_global_load_lds(g, (__attribute__((address_space(3))) void*)(uintptr_t)lds, 16, 0, 0);
 }
 
+// The same for bytes that one work group reads once (aux 2: non-temporal): streamed weights.
+__device__ __forceinline__ void lds_load16_nt(const bf16_t* g, bf16_t* lds) {
+  __builtin_amdgcn_global_load_lds(g, (__attribute__((address_space(3))) void*)(uintptr_t)lds, 16, 0, 2);
+}
+
 // LDS byte address of a pointer into the work group's shared memory (the low 32 bits of its
 // generic address; the LDS aperture is 4 GiB-aligned).
 __device__ __forceinline__ uint32_t lds_addr(const void* p) { return (uint32_t)(uintptr_t)p; }

@@ -1,4 +1,4 @@
-// Decoder layers for 9 to 64 token rows (a query, a follow-up turn, a short system prompt): every
+// Decoder layers for 9 to 128 token rows (a query, a follow-up turn, a short system prompt): every
 // projection streams its weights once from HBM, so the layer is priced by the weights' bytes and by
 // the launches between them. One call queues every kernel of every layer.
 //
@@ -24,7 +24,7 @@ constexpr int MID_TN = 64;        // features per tile
 constexpr int MID_BK = 128;       // K per unit
 constexpr int MID_THREADS = 256;  // 4 waves of 16 features
 constexpr int MID_CH = MID_BK / 8;
-constexpr int MID_MAX_ROWS = 64;
+constexpr int MID_MAX_ROWS = 128;
 constexpr int MID_MAX_HIDDEN = 16384;
 
 // How a projection's units are dealt: work group g takes units [g upg, (g + 1) upg).
@@ -79,7 +79,7 @@ __global__ __launch_bounds__(MID_THREADS) void mid_gemm_kernel(const MidGemmArgs
     const bf16_t* xp = a.x + ik * MID_BK;
     bf16_t* dst = smem + buf * ST::ELEMS;
 #pragma unroll
-    for (int q = 0; q < 4; ++q) lds_load16(wp + woff[q], dst + (q * 4 + wv) * 64 * 8);
+    for (int q = 0; q < 4; ++q) lds_load16_nt(wp + woff[q], dst + (q * 4 + wv) * 64 * 8);
 #pragma unroll
     for (int q = 0; q < MB; ++q) lds_load16(xp + xoff[q], dst + ST::W_ELEMS + (q * 4 + wv) * 64 * 8);
     if (++ik == a.p.ku) {
@@ -117,12 +117,13 @@ __global__ __launch_bounds__(MID_THREADS) void mid_gemm_kernel(const MidGemmArgs
         xf[s][b] = lds_read128<(ST::W_ELEMS + b * 16 * MID_BK) * 2>(addr[s] + so);
       });
     };
-    read(std::integral_constant<int, 0>{});
-    read(std::integral_constant<int, 1>{});
+    // reads of AHEAD steps in flight (the wait counter holds 15)
+    constexpr int AHEAD = 2 * (1 + MB) <= 15 ? 2 : 1;
+    static_for<AHEAD>([&](auto S) { read(S); });
     static_for<4>([&](auto S) {
       constexpr int s = decltype(S)::value;
-      if constexpr (s + 2 < 4) read(std::integral_constant<int, s + 2>{});
-      constexpr int after = (s + 2 < 4 ? 2 : 3 - s) * (1 + MB);
+      if constexpr (s + AHEAD < 4) read(std::integral_constant<int, s + AHEAD>{});
+      constexpr int after = (s + AHEAD < 4 ? AHEAD : 3 - s) * (1 + MB);
       lgkm_wait<after>(wf[s]);
 #pragma unroll
       for (int b = 0; b < MB; ++b) {
@@ -316,8 +317,8 @@ static bool mid_shape_ok(int64_t m, int64_t n, int64_t k) {
          k <= (1 << 20) && (n / MID_TN) * (k / MID_BK) <= (1 << 28);
 }
 
-// Pipeline depth and work groups per CU, by row blocks: what 160 KB of LDS holds.
-static int mid_stages(int mb) { return mb <= 2 ? 3 : 4; }
+// Pipeline stages by blocks of 16 rows, and (mid_plan) work groups per CU: what 160 KB of LDS holds.
+constexpr int mid_stages(int mb) { return mb <= 2 ? 3 : mb <= 6 ? 4 : 3; }
 static MidPlan mid_plan(int64_t m, int64_t n, int64_t k) {
   MidPlan p;
   p.tiles = (int)(n / MID_TN);
@@ -332,7 +333,8 @@ static size_t mid_part_bytes(const MidPlan& p, int64_t m) { return (size_t)(p.gr
 
 template <int MB>
 static void mid_launch(const MidGemmArgs& a, hipStream_t s) {
-  constexpr int NST = MB <= 2 ? 3 : 4;
+  constexpr int NST = mid_stages(MB);
+  static_assert(NST * MidStage<MB>::ELEMS * 2 * (MB <= 2 ? 2 : 1) <= 160 * 1024, "stages fit in LDS");
   hipLaunchKernelGGL((mid_gemm_kernel<MB, NST>), dim3(a.p.groups), dim3(MID_THREADS),
                      NST * MidStage<MB>::ELEMS * sizeof(bf16_t), s, a);
 }
@@ -347,10 +349,16 @@ static int mid_gemm(const bf16_t* x, const bf16_t* w, int64_t m, int64_t n, int6
   a.K = (int)k;
   a.p = mid_plan(m, n, k);
   *src = MidSrc{part, (int)m, a.p.ku, a.p.upg};
-  if (m <= 16) mid_launch<1>(a, s);
-  else if (m <= 32) mid_launch<2>(a, s);
-  else if (m <= 48) mid_launch<3>(a, s);
-  else mid_launch<4>(a, s);
+  switch ((m + 15) / 16) {
+    case 1: mid_launch<1>(a, s); break;
+    case 2: mid_launch<2>(a, s); break;
+    case 3: mid_launch<3>(a, s); break;
+    case 4: mid_launch<4>(a, s); break;
+    case 5: mid_launch<5>(a, s); break;
+    case 6: mid_launch<6>(a, s); break;
+    case 7: mid_launch<7>(a, s); break;
+    default: mid_launch<8>(a, s); break;
+  }
   return check_launch("mid gemm");
 }
 

@@ -151,7 +151,7 @@ def _mid_rows(P, n):
 
 
 def _layers_mid_rows(P, layers, h, delta, R, K, V):
-    """layer_forward of consecutive layers for 9 to 64 rows, in one library call."""
+    """layer_forward of consecutive layers for 9 to 128 rows, in one library call."""
     return _hip.mid_layers([P.layers[l] for l in layers], [(K[l], V[l]) for l in layers], h, delta, P.eps, P.hq, P.hkv,
                            P.hd, P.inter, R.cos, R.sin, R.rows, R.kend, P.scale, kseg=R.kseg, n_shared=R.n_shared)
 
