@@ -1143,7 +1143,9 @@ constexpr int DEC_MIN_SPLIT = 4 * DEC_BK;
 constexpr int ATT_LONG_MIN_TILES = 8;
 constexpr int64_t ATT_LONG_MAX_WGS = 1536;
 
-static SplitPlan plan_split(int64_t n, int hq, int hkv, int head_dim, int64_t t_cap) {
+// segments: the rows see the shared keys and their own segment only (kseg). Only fewer partials follow
+// from it, so the workspace is sized without.
+static SplitPlan plan_split(int64_t n, int hq, int hkv, int head_dim, int64_t t_cap, bool segments = false) {
   SplitPlan sp;
   sp.decode = false;
   if (n * (hq / hkv) <= DEC_ROWS) {
@@ -1178,8 +1180,16 @@ static SplitPlan plan_split(int64_t n, int hq, int hkv, int head_dim, int64_t t_
     const int64_t most = cus / base;  // splits
     if (most > 1) {
       len = (t_cap + most - 1) / most;
-      if (len < att_few_split_keys(head_dim)) len = att_few_split_keys(head_dim);
+      // a row of packed segments sees few of the cache's keys: as many slices as hold 512 (122 rows of
+      // two 0.5B documents, 186 keys: 16.2 us whole, 19.3 in two slices)
+      const int64_t coarse = t_cap / ATT_MIN_SPLIT_KEYS;
+      const int64_t least = !segments ? att_few_split_keys(head_dim) : coarse > 1 ? (t_cap + coarse - 1) / coarse : t_cap;
+      if (len < least) len = least;
       if (t_cap < len + 32) len = 0;
+      // More than four row tiles over a short cache (a small prefill: a row sees half the keys) stay
+      // whole where a split saves less than five tiles of a work group's loop, about the merge's
+      // launch (7B causal, 494 rows: 24.7 us whole, 28.8 split; 160 rows over 600 keys 29.9 and 25.5).
+      if (sp.tiles > 4 && t_cap < 2 * ATT_MIN_SPLIT_KEYS && (base > ATT_MANY_TILE_WGS / 2 || t_cap < len + 5 * bk)) len = 0;
     }
   } else if (base < ATT_TARGET_WGS && t_cap >= 2 * ATT_MIN_SPLIT_KEYS) {
     // Many row tiles with ragged key ranges (recompute rows sorted by position): about three
@@ -1389,7 +1399,7 @@ static int subset_attn_impl(const void* q, const void* k_cache, const void* v_ca
   a.hq = hq;
   a.hkv = hkv;
   a.G = hq / hkv;
-  SplitPlan sp = plan_split(n, hq, hkv, head_dim, t_cap);
+  SplitPlan sp = plan_split(n, hq, hkv, head_dim, t_cap, kseg != nullptr);
   const size_t need = split_ws_bytes(sp, hkv, head_dim);
   if (need && (!ws || ws_bytes < need)) {  // no workspace: one pass per row tile (decode: one slice)
     sp.nsplit = 1;
