@@ -122,17 +122,30 @@ def _freq(inv_freq):
 
 # ------------------------------------------------------------------------------------------- (a)
 
+def _delta_cos_sin(inv_freq, deltas):
+    """cos and sin of fp32(delta) * inv_freq, fp32 [n, hd/2] on the host, with the vectorised torch ops of
+    the reference's rotary embedding (its fp32 outer product has one term per element, so a broadcast
+    product gives the same bits)."""
+    f = inv_freq.detach().to("cpu", torch.float32)
+    if not deltas:
+        return f.new_empty(0, f.numel()), f.new_empty(0, f.numel())
+    ang = torch.outer(torch.frombuffer((c_float * len(deltas))(*deltas), dtype=torch.float32), f)
+    return ang.cos(), ang.sin()
+
+
 def delta_table_host(inv_freq, deltas):
     """fp32 [n, hd/2, 2] (cos, sin) of fp32(delta) * inv_freq on the host, computed with the same
-    torch ops as the reference's rotary embedding (fp32 outer product, then cos / sin)."""
-    pos = torch.tensor([int(d) for d in deltas], dtype=torch.int64)
-    freqs = (inv_freq.detach().to("cpu", torch.float32)[:, None] @ pos[None, :].float()).transpose(0, 1)
-    return torch.stack([freqs.cos(), freqs.sin()], dim=-1).contiguous()
+    torch ops as the reference's rotary embedding (fp32 product, then cos / sin)."""
+    return torch.stack(_delta_cos_sin(inv_freq, [int(d) for d in deltas]), dim=-1)
 
 
 def delta_table(inv_freq, deltas, device):
-    """delta_table_host, moved to `device`."""
-    return delta_table_host(inv_freq, deltas).pin_memory().to(device, non_blocking=True)
+    """delta_table_host on `device`, written straight into pinned memory (stacking, then pinning a copy
+    of it, made half of a small launch's host time)."""
+    deltas = [int(d) for d in deltas]
+    t = torch.empty(len(deltas), inv_freq.numel(), 2, dtype=torch.float32, pin_memory=True)
+    torch.stack(_delta_cos_sin(inv_freq, deltas), dim=-1, out=t)
+    return t.to(device, non_blocking=True)
 
 
 def rope_assemble(sources, dst_k, dst_v, inv_freq, layer_lo=0, layer_hi=None, table=None):
@@ -150,16 +163,21 @@ def rope_assemble(sources, dst_k, dst_v, inv_freq, layer_lo=0, layer_hi=None, ta
         raise ValueError("dst_k must be [L, 1, kv, t_cap, hd]")
     layer_hi = L if layer_hi is None else layer_hi
     arr = (Src * max(1, len(sources)))()
+    lead = (L, 1, kv)
     for i, (K, V, off, delta) in enumerate(sources):
-        _need(K, f"source {i} K")
-        if K.shape[:3] != (L, 1, kv) or K.shape[-1] != hd:
+        if not (K.is_cuda and K.dtype is torch.bfloat16 and K.is_contiguous()):
+            _need(K, f"source {i} K")
+        shape = K.shape
+        if shape[:3] != lead or shape[-1] != hd:
             raise ValueError(f"source {i}: shape {tuple(K.shape)} does not match cache {tuple(dst_k.shape)}")
+        vp = 0
         if dst_v is not None:
-            _need(V, f"source {i} V")
-            if V.shape != K.shape:
+            if not (V.is_cuda and V.dtype is torch.bfloat16 and V.is_contiguous()):
+                _need(V, f"source {i} V")
+            if V.shape != shape:
                 raise ValueError(f"source {i}: V shape {tuple(V.shape)} differs from K {tuple(K.shape)}")
-        vp = V.data_ptr() if dst_v is not None else 0
-        arr[i] = Src(K.data_ptr(), vp, K.shape[-2], int(off), int(delta))
+            vp = V.data_ptr()
+        arr[i] = (K.data_ptr(), vp, shape[-2], int(off), int(delta))
     if table is None:
         table = delta_table(inv_freq, [s[3] for s in sources], dst_k.device)
     if table.shape != (len(sources), hd // 2, 2) or table.dtype != torch.float32 or not table.is_cuda:
