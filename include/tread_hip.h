@@ -202,6 +202,21 @@ size_t tread_skinny_silu_workspace_bytes(int64_t m, int64_t n, int64_t inter);
 int tread_skinny_silu_linear_bf16(const void* gate_up, int64_t m, int64_t inter, const void* weight, int64_t n, void* y,
                                   void* ws, size_t ws_bytes, tread_stream_t stream);
 
+/* Linear layer of any number of token rows: y[m, n] = x[m, k] . weight[n, k]^T (+ bias[n]), bf16, fp32
+ * accumulation, one bf16 rounding (as F.linear); all contiguous and 16-byte aligned, n a multiple of
+ * 8, k of 64. The tiles of the last, partial round over the GPU are cut along k when ws (device) holds
+ * tread_linear_workspace_bytes(m, n, k) bytes; with ws NULL or too small the call still succeeds.
+ * linear_swiglu: y[m, inter] = bf16(bf16(silu(g)) * u) with [g | u] = x . wgu^T (wgu: [2 inter, k], gate
+ * rows then up rows; g and u rounded to bf16 first, silu_mul's roundings; inter a multiple of 8), without
+ * the [m, 2 inter] intermediate; its workspace is that of n = 2 inter. Replaces the MLP's
+ * act_fn(gate_proj(x)) * up_proj(x) (transformers Qwen2MLP at tread/blend.py:103,111-113).
+ */
+size_t tread_linear_workspace_bytes(int64_t m, int64_t n, int64_t k);
+int tread_linear_bf16(const void* x, const void* weight, const void* bias, int64_t m, int64_t n, int64_t k, void* y,
+                      void* ws, size_t ws_bytes, tread_stream_t stream);
+int tread_linear_swiglu_bf16(const void* x, const void* wgu, int64_t m, int64_t inter, int64_t k, void* y, void* ws,
+                             size_t ws_bytes, tread_stream_t stream);
+
 /* Linear layer of up to 128 token rows: y[m, n] = x[m, k] . weight[n, k]^T (+ bias[n]), bf16, fp32
  * accumulation, one bf16 rounding (as F.linear); x, y and weight contiguous and 16-byte aligned, n a
  * multiple of 64, k of 128. The weights are streamed once, cut into equal spans over the GPU; the

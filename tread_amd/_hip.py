@@ -58,6 +58,9 @@ _SIGS = {
                                               c_void, c_void]),
     "tread_skinny_silu_workspace_bytes": (c_size, [c_i64, c_i64, c_i64]),
     "tread_skinny_silu_linear_bf16": (c_int, [c_void, c_i64, c_i64, c_void, c_i64, c_void, c_void, c_size, c_void]),
+    "tread_linear_workspace_bytes": (c_size, [c_i64, c_i64, c_i64]),
+    "tread_linear_bf16": (c_int, [c_void, c_void, c_void, c_i64, c_i64, c_i64, c_void, c_void, c_size, c_void]),
+    "tread_linear_swiglu_bf16": (c_int, [c_void, c_void, c_i64, c_i64, c_i64, c_void, c_void, c_size, c_void]),
     "tread_mid_linear_workspace_bytes": (c_size, [c_i64, c_i64, c_i64]),
     "tread_mid_linear_bf16": (c_int, [c_void, c_void, c_void, c_i64, c_i64, c_i64, c_void, c_void, c_size, c_void]),
     "tread_mid_layers_workspace_bytes": (c_size, [c_i64, c_int, c_int, c_int, c_int, c_int, c_i64]),
@@ -373,6 +376,44 @@ def skinny_silu_linear(gate_up, weight):
     ws = torch.empty(wsb, dtype=torch.uint8, device=gate_up.device) if wsb else None
     _check("tread_skinny_silu_linear_bf16", lib().tread_skinny_silu_linear_bf16(
         _ptr(gate_up), m, inter, _ptr(weight), n, _ptr(y), _ptr(ws), wsb, _stream()))
+    return y
+
+
+def _linear_ws(m, n, k, device):
+    wsb = lib().tread_linear_workspace_bytes(m, n, k)
+    return (torch.empty(wsb, dtype=torch.uint8, device=device) if wsb else None), wsb
+
+
+def linear(x, weight, bias=None):
+    """y = x @ weight.T (+ bias) for many rows x [m, k] (n % 8 == 0, k % 64 == 0)."""
+    _need(x, "x")
+    _need(weight, "weight")
+    if bias is not None:
+        _need(bias, "bias")
+    m, k = x.shape
+    n = weight.shape[0]
+    if weight.shape[1] != k or (bias is not None and bias.numel() != n):
+        raise ValueError(f"linear: x {tuple(x.shape)} weight {tuple(weight.shape)}")
+    y = torch.empty(m, n, dtype=x.dtype, device=x.device)
+    ws, wsb = _linear_ws(m, n, k, x.device)
+    _check("tread_linear_bf16", lib().tread_linear_bf16(_ptr(x), _ptr(weight), _ptr(bias), m, n, k, _ptr(y), _ptr(ws),
+                                                       wsb, _stream()))
+    return y
+
+
+def linear_swiglu(x, wgu):
+    """bf16(silu(g)) * u with [g | u] = x @ wgu.T (wgu [2 inter, k]) for many rows x [m, k]: silu_mul's
+    roundings without the [m, 2 inter] intermediate."""
+    _need(x, "x")
+    _need(wgu, "wgu")
+    m, k = x.shape
+    n = wgu.shape[0]
+    if wgu.shape[1] != k or n % 16:
+        raise ValueError(f"linear_swiglu: x {tuple(x.shape)} wgu {tuple(wgu.shape)}")
+    y = torch.empty(m, n // 2, dtype=x.dtype, device=x.device)
+    ws, wsb = _linear_ws(m, n, k, x.device)
+    _check("tread_linear_swiglu_bf16", lib().tread_linear_swiglu_bf16(_ptr(x), _ptr(wgu), m, n // 2, k, _ptr(y),
+                                                                     _ptr(ws), wsb, _stream()))
     return y
 
 

@@ -53,6 +53,45 @@ def _gate_up(x, w, split):
     return y
 
 
+# Where the library's own GEMM kernels (csrc/gemm.hip, 256 x 256 tiles, one per CU and round) beat the
+# BLAS library's untuned choice, measured on MI355X:
+# - gate|up + SiLU gating in one kernel up to a hidden size of 1 024 and from two rounds of tiles on: 18 row
+#   counts from 3 350 to 8 977 of a 0.5B shape (896 -> 2 x 4 864), 0.95-1.26x, 1.11x in the mean (8 000 rows:
+#   179 us for the GEMM and the gating, 153 us fused); below two rounds the half-empty second one loses
+#   (1 632 rows: 45 and 59 us), and at hidden sizes of 1 536 and more the library's faster inner loop
+#   makes up for the gating pass (7B, 6 432 rows: 1 403 and 1 560 us).
+# - a down projection of 16 384 and more inputs, from one round of tiles up to two: 16 row counts from
+#   4 693 to 7 900 of the 7B shape (18 944 -> 3 584), 1.35x in the mean (6 432 rows: 1 153 and 748 us).
+#   The library's time jumps with its choice of tile there: at 5 489, 5 688 and 6 882 rows it is 10-17 %
+#   faster than this kernel, elsewhere 26-75 % slower. Below one round it is ahead at 1 632, 3 219 and
+#   4 300-4 500 rows, behind at most others; from two rounds on (70B: 28 672 -> 8 192) mostly ahead.
+GEMM_TILE, GEMM_ROUND = 256, 256
+
+
+def _rounds(n, features):
+    return -(-n // GEMM_TILE) * -(-features // GEMM_TILE) / GEMM_ROUND
+
+
+def _swiglu_pays(n, features, k):
+    return k <= 1024 and k % 64 == 0 and features % 16 == 0 and _rounds(n, features) >= 2
+
+
+def _linear_pays(n, features, k):
+    return k >= 16384 and k % 64 == 0 and features % 8 == 0 and 1 < _rounds(n, features) < 2
+
+
+def _mlp(x, lw, split):
+    """The MLP of the normed rows x [n, H]: gate|up, SiLU gating, down."""
+    tuned = torch.cuda.tunable.is_enabled()  # the caller routes the GEMMs through measured solutions
+    if not tuned and _swiglu_pays(x.shape[0], lw.wgu.shape[0], lw.wgu.shape[1]):
+        m = _hip.linear_swiglu(x, lw.wgu)
+    else:
+        m = _hip.silu_mul(_gate_up(x, lw.wgu, split))
+    if not tuned and _linear_pays(m.shape[0], lw.wd.shape[0], lw.wd.shape[1]):
+        return _hip.linear(m, lw.wd)
+    return F.linear(m, lw.wd)
+
+
 def make_rows(P, rows, pos=None, kseg=None, n_shared=0):
     """RoPE tables for `pos` (default: rows) and causal key ends = rows."""
     rows = rows.to(torch.int64).contiguous()
@@ -84,8 +123,7 @@ def layer_forward(P, l, h, delta, R: Rows, K, V, kv_only=False):
     o = _hip.subset_attn(q, K[l], V[l], R.kend, hq, hkv, hd, P.scale, kseg=R.kseg, n_shared=R.n_shared)
     a = F.linear(o, lw.wo)
     h, x = _hip.add_rmsnorm(h, lw.ln2, P.eps, delta=a)
-    m = _hip.silu_mul(_gate_up(x, lw.wgu, R.gemm_split))
-    return h, F.linear(m, lw.wd)
+    return h, _mlp(x, lw, R.gemm_split)
 
 
 # A layer of at most FEW_ROWS rows (a decoding step, a short query) runs its projections on the
