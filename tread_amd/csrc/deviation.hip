@@ -8,7 +8,7 @@
 //
 // Select: one work group of 1024 threads stages the 16-bit ordered score keys in LDS (up to 64 Ki
 // candidates), runs a two-pass radix select over them (high byte, then low byte, into a 256-bin LDS
-// histogram replicated so that one wave's atomics spread over 16 words), and an order-preserving
+// histogram replicated so that one wave's atomics spread over 16 or 64 words), and an order-preserving
 // compaction, so the selected candidate indices come out ascending.
 #include "common.h"
 #include "../../include/tread_hip.h"
@@ -112,7 +112,13 @@ constexpr int SEL_THREADS = 1024;
 constexpr int SEL_WAVES = SEL_THREADS / 64;
 constexpr int64_t SEL_LDS_KEYS = 65536;  // candidates whose keys are staged in LDS (128 KiB)
 constexpr int64_t SEL_MAX_N = 1 << 20;   // keeps every 16-bit histogram counter at or below 2^15
-constexpr int SEL_HROWS = 16, SEL_HSTRIDE = 257;  // histogram rows; odd stride spreads rows over banks
+constexpr int SEL_HSTRIDE = 257;  // words of a histogram row; odd, so that rows spread over the banks
+// From SEL_WIDE_FROM to SEL_WIDE_TO keys the histogram has a row per lane (66 KB beside the keys), so that no
+// two lanes of an atomic hit the same word: request scores cluster in one or two high-byte bins, and with
+// 16 rows four lanes of each instruction serialise (32 000 keys: 22.0 us with 16 rows merged by a thread per
+// bin, 19.4 with 64 merged by four). Clearing 64 rows costs fewer keys more than that (1 000: 7.1 and 8.2 us),
+// and more keys leave no room for them.
+constexpr int64_t SEL_WIDE_FROM = 12288, SEL_WIDE_TO = 40960;
 
 __device__ __forceinline__ uint32_t lanes_below(uint64_t mask) {  // set bits of mask in lanes < this lane
   return __builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mask, 0u));
@@ -155,18 +161,19 @@ __device__ __forceinline__ void find_bin(const uint32_t* tot, uint32_t above, in
   }
 }
 
+template <int HROWS>
 __global__ __launch_bounds__(SEL_THREADS) void topk_select_kernel(const bf16_t* __restrict__ score, int64_t n,
                                                                   int64_t k, int64_t* __restrict__ sel) {
-  extern __shared__ uint16_t keys[];  // n ordered keys when n <= SEL_LDS_KEYS
-  // One 256-bin histogram shared by all waves, replicated over 16 rows x 2 halves so that the 64
-  // lanes of one atomic instruction hit 16 different words (lane l: row (l / 2) % 16, 16-bit half
-  // l % 2): request scores cluster in few bins, and same-word atomics of one wave serialise.
-  __shared__ uint32_t hist[SEL_HROWS * SEL_HSTRIDE];
+  // one 256-bin histogram shared by all waves in HROWS replicas, then the n ordered keys when
+  // n <= SEL_LDS_KEYS. HROWS 64: lane l counts in row l; 16: in row (l / 2) % 16, 16-bit half l % 2.
+  extern __shared__ __align__(16) uint32_t hist[];
+  uint16_t* const keys = reinterpret_cast<uint16_t*>(hist + HROWS * SEL_HSTRIDE);
   __shared__ uint32_t tot[256];
   __shared__ uint32_t s_thr, s_above, s_cnt_g[SEL_WAVES], s_cnt_t[SEL_WAVES];
   const int tid = threadIdx.x, wv = tid >> 6, lane = tid & 63;
-  uint32_t* const hrow = hist + ((lane >> 1) & (SEL_HROWS - 1)) * SEL_HSTRIDE;
-  const uint32_t hinc = (lane & 1) ? 0x10000u : 1u;
+  static_assert(HROWS == 64 || HROWS == 16, "a row per lane, or per four lanes in halves");
+  uint32_t* const hrow = hist + (HROWS == 64 ? lane : (lane >> 1) & 15) * SEL_HSTRIDE;
+  const uint32_t hinc = HROWS == 16 && (lane & 1) ? 0x10000u : 1u;
   const bool staged = n <= SEL_LDS_KEYS;
   // keys j .. j + 7 (j a multiple of 8), two per dword, low half first; keys at n and beyond are
   // unspecified and masked by the callers
@@ -182,18 +189,19 @@ __global__ __launch_bounds__(SEL_THREADS) void topk_select_kernel(const bf16_t* 
     return kk;
   };
   auto clear = [&]() {
-    for (int b = tid; b < SEL_HROWS * SEL_HSTRIDE; b += SEL_THREADS) hist[b] = 0;
+    for (int b = tid; b < HROWS * SEL_HSTRIDE; b += SEL_THREADS) hist[b] = 0;
   };
-  auto merge = [&]() {
-    if (tid < 256) {
-      uint32_t t = 0;
+  auto merge = [&]() {  // four threads per bin, a quarter of the rows each
+    const int bin = tid >> 2, part = tid & 3;
+    uint32_t t = 0;
 #pragma unroll
-      for (int r = 0; r < SEL_HROWS; ++r) {
-        const uint32_t x = hist[r * SEL_HSTRIDE + tid];
-        t += (x & 0xffffu) + (x >> 16);
-      }
-      tot[tid] = t;
+    for (int r = 0; r < HROWS / 4; ++r) {
+      const uint32_t x = hist[(part * (HROWS / 4) + r) * SEL_HSTRIDE + bin];
+      t += HROWS == 64 ? x : (x & 0xffffu) + (x >> 16);
     }
+    t += __shfl_xor(t, 1);
+    t += __shfl_xor(t, 2);
+    if (part == 0) tot[bin] = t;
   };
   // pass 1: stage the keys, histogram of the high byte. 16-byte loads, UNR of them in flight per
   // thread, when the scores are 16-byte aligned; a scalar loop for the rest.
@@ -362,8 +370,13 @@ extern "C" int tread_topk_select_bf16(const void* score, int64_t n, int64_t k, i
   if (k == 0) return 0;
   if (!score || !sel_out) return fail(TREAD_EINVAL, "topk_select: null pointer");
   if (n > SEL_MAX_N) return fail(TREAD_ERANGE, "topk_select: n=%lld above %lld candidates", (long long)n, (long long)SEL_MAX_N);
-  const size_t lds = n <= SEL_LDS_KEYS ? (size_t)(n + 7) / 8 * 16 : 0;  // whole 16-byte groups of keys
-  hipLaunchKernelGGL(topk_select_kernel, dim3(1), dim3(SEL_THREADS), lds, (hipStream_t)stream, (const bf16_t*)score, n,
-                     k, sel_out);
+  const size_t keys = n <= SEL_LDS_KEYS ? (size_t)(n + 7) / 8 * 16 : 0;  // whole 16-byte groups of keys
+  auto hist = [](int rows) { return (size_t)rows * SEL_HSTRIDE * sizeof(uint32_t); };
+  if (n >= SEL_WIDE_FROM && n <= SEL_WIDE_TO)
+    hipLaunchKernelGGL(topk_select_kernel<64>, dim3(1), dim3(SEL_THREADS), hist(64) + keys, (hipStream_t)stream,
+                       (const bf16_t*)score, n, k, sel_out);
+  else
+    hipLaunchKernelGGL(topk_select_kernel<16>, dim3(1), dim3(SEL_THREADS), hist(16) + keys, (hipStream_t)stream,
+                       (const bf16_t*)score, n, k, sel_out);
   return check_launch("topk_select");
 }
