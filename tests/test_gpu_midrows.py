@@ -1,4 +1,4 @@
-"""Decoder layers of 9 to 128 rows (tread_mid_layers_bf16) and their weight-streaming projection."""
+"""Decoder layers of 3 to 128 rows (tread_mid_layers_bf16) and their weight-streaming projection."""
 import pytest
 import torch
 
@@ -34,7 +34,7 @@ def _layer_inputs(cfg, m, t_cap, seed):
     return blend.prepared(model), bf(m, cfg.hidden_size), bf(m, cfg.hidden_size, scale=0.1), bf(*shape), bf(*shape)
 
 
-@pytest.mark.parametrize("m,hd,form", [(9, 64, "tail"), (16, 128, "docs"), (17, 64, "pads"), (33, 128, "tail"),
+@pytest.mark.parametrize("m,hd,form", [(3, 128, "tail"), (9, 64, "tail"), (16, 128, "docs"), (17, 64, "pads"), (33, 128, "tail"),
                                        (64, 64, "docs"), (65, 128, "pads"), (128, 64, "tail")])
 def test_mid_layers_match_the_separate_launches(m, hd, form, monkeypatch):
     """Two layers in one call against the path for many rows (library GEMMs and separate launches):
@@ -54,7 +54,7 @@ def test_mid_layers_match_the_separate_launches(m, hd, form, monkeypatch):
     K2, V2 = K.clone(), V.clone()
     with torch.inference_mode():
         a = forward.run_layers(P, h, d, R, K.unbind(0), V.unbind(0), range(2))
-        monkeypatch.setattr(forward, "_mid_rows", lambda P, n: False)
+        monkeypatch.setattr(forward, "_mid_rows", lambda *a: False)
         b = forward.run_layers(P, h, d, R, K2.unbind(0), V2.unbind(0), range(2))
     for x, y in ((a[0], b[0]), (a[1], b[1]), (K, K2), (V, V2)):
         # bf16 rounding of every intermediate, in another order: 2^-8 each, a dozen of them a layer
@@ -65,24 +65,16 @@ def test_mid_layers_match_the_separate_launches(m, hd, form, monkeypatch):
     assert torch.equal(K[..., keep, :], K2[..., keep, :]) and torch.equal(V[..., keep, :], V2[..., keep, :])
 
 
-@pytest.mark.parametrize("hd,G,hkv", [(128, 7, 4), (64, 7, 2)])
-@pytest.mark.parametrize("n,keys", [(37, 191), (37, 223), (37, 224), (37, 1500), (160, 600), (300, 700), (160, 9000)])
-def test_query_attention_slices_match_fp64(hd, G, hkv, n, keys):
-    """Key slices at the edges of the split rule: one slice and two, whole and cut row tiles, up to one
-    work group per CU."""
-    g = torch.Generator().manual_seed(keys + n)
-    q = torch.randn(n, G * hkv, hd, generator=g).to(torch.bfloat16)
-    K = (2 * torch.randn(1, hkv, keys, hd, generator=g)).to(torch.bfloat16)
-    V = torch.randn(1, hkv, keys, hd, generator=g).to(torch.bfloat16)
-    kend = torch.randperm(keys, generator=g)[:n] if n <= keys else torch.arange(n).clamp(max=keys - 1)
-    kend = kend.sort().values if n <= keys else kend
-    out = _hip.subset_attn(q.to(DEV), K.to(DEV), V.to(DEV), kend.to(DEV), G * hkv, hkv, hd, hd ** -0.5).cpu().double()
-    see = torch.arange(keys)[None] <= kend[:, None]
-    for h in range(hkv):
-        s = torch.einsum("ngd,kd->ngk", q[:, h * G:(h + 1) * G].double(), K[0, h].double()) * hd ** -0.5
-        p = s.masked_fill(~see[:, None], float("-inf")).softmax(-1)
-        ref = (p @ V[0, h].double()).reshape(n, -1)
-        got = out.view(n, hkv, -1)[:, h]
-        # bf16 rounding of the scaled q (scores off by 2^-9 of their size, up to about 10 here), of P and
-        # of the result
-        assert (got - ref).norm() <= 1.2e-2 * ref.norm()
+def test_mid_layers_leave_strided_weights_to_the_library():
+    """A down projection stored transposed: the call is taken as before."""
+    cfg = ModelConfig(512, 384, 1, 6, 2, 64, 640)
+    P, h, d, K, V = _layer_inputs(cfg, 20, 100, seed=2)
+    rows = torch.arange(40, 60, device=DEV)
+    R = forward.make_rows(P, rows)
+    with torch.inference_mode():
+        a = forward.run_layers(P, h, d, R, K.unbind(0), V.unbind(0), range(1))
+        P.layers[0].wd = P.layers[0].wd.t().contiguous().t()
+        assert not forward._mid_rows(P, 20, [0])
+        b = forward.run_layers(P, h, d, R, K.unbind(0), V.unbind(0), range(1))
+    for x, y in zip(a, b):  # bf16 rounding of every intermediate, in another order
+        assert (x.float() - y.float()).norm() <= 0.02 * y.float().norm()

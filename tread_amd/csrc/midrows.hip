@@ -1,4 +1,4 @@
-// Decoder layers for 9 to 128 token rows (a query, a follow-up turn, a short system prompt): every
+// Decoder layers for 3 to 128 token rows (a query, a follow-up turn, a short system prompt): every
 // projection streams its weights once from HBM, so the layer is priced by the weights' bytes and by
 // the launches between them. One call queues every kernel of every layer.
 //

@@ -83,11 +83,11 @@ def _linear_pays(n, features, k):
 def _mlp(x, lw, split):
     """The MLP of the normed rows x [n, H]: gate|up, SiLU gating, down."""
     tuned = torch.cuda.tunable.is_enabled()  # the caller routes the GEMMs through measured solutions
-    if not tuned and _swiglu_pays(x.shape[0], lw.wgu.shape[0], lw.wgu.shape[1]):
+    if not tuned and _swiglu_pays(x.shape[0], *lw.wgu.shape) and _streamable(lw.wgu):
         m = _hip.linear_swiglu(x, lw.wgu)
     else:
         m = _hip.silu_mul(_gate_up(x, lw.wgu, split))
-    if not tuned and _linear_pays(m.shape[0], lw.wd.shape[0], lw.wd.shape[1]):
+    if not tuned and _linear_pays(m.shape[0], *lw.wd.shape) and _streamable(lw.wd):
         return _hip.linear(m, lw.wd)
     return F.linear(m, lw.wd)
 
@@ -106,10 +106,10 @@ def layer_forward(P, l, h, delta, R: Rows, K, V, kv_only=False):
     Returns (h, delta) entering layer l+1, or (h, None) when kv_only (k/v spliced, nothing else)."""
     lw = P.layers[l]
     hq, hkv, hd = P.hq, P.hkv, P.hd
+    if not kv_only and _mid_rows(P, h.shape[0], (l,)):
+        return _layers_mid_rows(P, [l], h, delta, R, K, V)
     if not kv_only and _few_rows(P, lw, h.shape[0]):
         return _layer_few_rows(P, l, lw, h, delta, R, K, V)
-    if not kv_only and _mid_rows(P, h.shape[0]):
-        return _layers_mid_rows(P, [l], h, delta, R, K, V)
     h, x = _hip.add_rmsnorm(h, lw.ln1, P.eps, delta=delta)
     n = h.shape[0]
     if kv_only:
@@ -126,15 +126,13 @@ def layer_forward(P, l, h, delta, R: Rows, K, V, kv_only=False):
     return h, _mlp(x, lw, R.gemm_split)
 
 
-# A layer of at most FEW_ROWS rows (a decoding step, a short query) runs its projections on the
-# weight-streaming skinny kernels, which beat the library GEMM there on MI355X. The kernels with
+# A layer of one or two rows (a decoding step), and of up to FEW_ROWS where mid_layers does not take it, runs
+# its projections on the weight-streaming skinny kernels, which beat the library GEMM there on MI355X. The kernels with
 # the norm (or the SiLU gating) fused in front save a launch but redo that prologue in every work
 # group for every row; measured on MI355X they win up to NORM_FUSED_ROWS rows (norm) and
 # SILU_FUSED_ROWS rows (SiLU) and lose beyond (at 8 rows the norm-fused lm_head takes twice the
-# time of RMSNorm + skinny kernel). Fused or not, the results are the same bits. Up to the skinny
-# kernels' 32 rows they lose: a 32-row query forward over a 7B-shaped model's cache of 32k rows
-# took 8.5 ms on them against 6.5 ms on the library GEMMs (the whole request without recompute),
-# over a 0.5B-shaped one's 1k and 8k rows 2.8 and 2.9 ms against 2.2 and 2.4 ms.
+# time of RMSNorm + skinny kernel). Fused or not, the results are the same bits. Up to the skinny kernels' 32
+# rows they lose (a 7B gate|up of 16 rows takes 65.8 us against 46.1 on the kernels of mid_layers).
 FEW_ROWS = 8
 NORM_FUSED_ROWS = 2
 SILU_FUSED_ROWS = 4
@@ -184,12 +182,34 @@ def _layer_few_rows(P, l, lw, h, delta, R, K, V):
     return h, _silu_linear(gu, lw.wd)
 
 
-def _mid_rows(P, n):
-    return FEW_ROWS < n <= _hip.MID_MAX_ROWS and _hip.mid_layers_ok(n, P.H, P.hq, P.hkv, P.hd, P.inter)
+# From three to 128 rows the layers run in one library call on the weight-streaming kernels of
+# csrc/midrows.hip (other widths and weights: the skinny kernels up to FEW_ROWS rows, then the library). A
+# decoding step of 3 and 8 tokens over a few layers and the lm_head, skinny / those kernels, in us: 0.5B over 8 000
+# keys 277 / 254 and 305 / 267, 1.5B over 16 000 400 / 343 and 434 / 355, 7B over 32 000 666 / 560 and 689 / 564; two
+# rows are left to the fused skinny kernels (0.5B 218 / 244, 7B 599 / 551). Four projections of a layer, library GEMMs / those kernels, in us: 7B 32 rows 193 / 109
+# (down alone 109 / 30), 64 rows 183 / 127, 128 rows 210 / 176; 0.5B 32 rows 39 / 33, 64 rows 44 / 38, 128 rows
+# 41 / 49, where the consumers of the partial sums still save a launch each and a separate call its host time.
+MID_MIN_ROWS = 3
+
+
+def _mid_rows(P, n, layers):
+    return (MID_MIN_ROWS <= n <= _hip.MID_MAX_ROWS and _hip.mid_layers_ok(n, P.H, P.hq, P.hkv, P.hd, P.inter)
+            and all(_streamable(w) for l in layers for w in _weights(P.layers[l])))
+
+
+def _weights(lw):
+    ws = (lw.ln1, lw.wqkv, lw.wo, lw.ln2, lw.wgu, lw.wd)
+    return ws if lw.bqkv is None else ws + (lw.bqkv,)
+
+
+def _streamable(w):
+    """What the kernels that read 16 bytes a lane take; other weights (a model's own views) stay with the
+    library."""
+    return w.is_contiguous() and w.data_ptr() % 16 == 0
 
 
 def _layers_mid_rows(P, layers, h, delta, R, K, V):
-    """layer_forward of consecutive layers for 9 to 128 rows, in one library call."""
+    """layer_forward of consecutive layers for 3 to 128 rows, in one library call."""
     return _hip.mid_layers([P.layers[l] for l in layers], [(K[l], V[l]) for l in layers], h, delta, P.eps, P.hq, P.hkv,
                            P.hd, P.inter, R.cos, R.sin, R.rows, R.kend, P.scale, kseg=R.kseg, n_shared=R.n_shared)
 
@@ -201,7 +221,7 @@ def run_layers(P, h, delta, R, K, V, layers, kv_only_last=False, hook=None, keep
     row's k/v is in place; the result is those rows' (h, delta)."""
     layers = list(layers)
     whole = layers[:-1] if kv_only_last else layers
-    if hook is None and whole and _mid_rows(P, h.shape[0]):  # nothing waits between layers
+    if hook is None and whole and _mid_rows(P, h.shape[0], whole):  # nothing waits between layers
         h, delta = _layers_mid_rows(P, whole, h, delta, R, K, V)
         layers = layers[len(whole):]
     for j, l in enumerate(layers):
