@@ -322,8 +322,8 @@ __global__ __launch_bounds__(GEMM_THREADS) void gemm_kernel(const GemmArgs a) {
   vm_wait<0>();  // the loads past the stream's end
 }
 
-// Adds the K slices of the last round's tiles in order and finishes them: one wave per wave of the
-// tile's work group, blockIdx.x = tile * 8 + wave.
+// Adds the K slices of the last round's tiles in order and finishes them: one wave per 64 features x 32 rows
+// of a tile (a 32-row block of one of the tile's waves: tile, wave, block from blockIdx.x).
 template <bool SWIGLU>
 __global__ __launch_bounds__(64) void gemm_reduce_kernel(const GemmArgs a, int first) {
   const int c0 = blockIdx.x & 3, wv = (blockIdx.x >> 2) % GEMM_WAVES, t = (blockIdx.x >> 2) / GEMM_WAVES;
